@@ -210,7 +210,7 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
                 const double px = s.px[p], py = s.py[p], z = s.pz[p];
                 const double q = DIFF == OHX_DIFF_FRESNEL ? s.q[p] : 0.0;
                 int4 ib;
-                rank = taken_rank<DIFF, double>(g, px, py, z, q, s.kamp[p], b, x0, y0, ib);
+                rank = taken_rank<DIFF, double>(g, px, py, z, q, s.cyc0[p], s.kamp[p], b, x0, y0, ib);
                 if (rank == 0) sm.left[0] = 1;
                 else if (DIFF == OHX_DIFF_RS && edge_lines(b, ib, x0, cx1, y0, ry1)) sm.left[1] = 1;
                 bb = box_bits(ib, x0, y0);

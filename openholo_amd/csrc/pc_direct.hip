@@ -257,10 +257,11 @@ __device__ inline double* slot_fp64(float2* row_entry) { return reinterpret_cast
 // The matrix product left the pair of a point (box b) and the tile that holds
 // pixel (x0, y0)
 template <typename T>
-__device__ inline bool left_pair(const Geometry& g, double px, double py, double z, double kamp, int4 b, int x0, int y0)
+__device__ inline bool left_pair(const Geometry& g, double px, double py, double z, double cyc0, double kamp, int4 b,
+                                 int x0, int y0)
 {
     int4 ib;
-    return dgemm::taken_rank<OHX_DIFF_RS, T>(g, px, py, z, 0.0, kamp, b, x0 / dgemm::GW * dgemm::GW,
+    return dgemm::taken_rank<OHX_DIFF_RS, T>(g, px, py, z, 0.0, cyc0, kamp, b, x0 / dgemm::GW * dgemm::GW,
                                       y0 / dgemm::Kind<T>::GH * dgemm::Kind<T>::GH, ib) == 0;
 }
 
@@ -315,7 +316,7 @@ __device__ __attribute__((always_inline)) inline void rest_tile(DirectSmem& sm, 
         if (tid < PCH && p < p_end && !skip) {
             b = s.box[p];
             if (b.x < cx1 && b.y > x0 && b.z < ry1 && b.w > y0 &&
-                (all || left_pair<float>(g, s.px[p], s.py[p], s.pz[p], s.kamp[p], b, x0, y0))) {
+                (all || left_pair<float>(g, s.px[p], s.py[p], s.pz[p], s.cyc0[p], s.kamp[p], b, x0, y0))) {
                 const bool full = b.x <= x0 && b.y >= cx1 && b.z <= y0 && b.w >= ry1;
                 px = s.px[p];
                 py = s.py[p];
@@ -332,8 +333,9 @@ __device__ __attribute__((always_inline)) inline void rest_tile(DirectSmem& sm, 
                                     2.0 * vmax * fabs(dyc) + (double)vmax * vmax;
                 const double e = nmax / rc2;
                 // third-order phase term e^3 r_c/(16 lambda) and second-order
-                // amplitude term e^2 must be negligible
-                const bool series_ok = e * e * e * rc * g.inv_lambda < 16 * 2e-7 && e * e < 1e-7 &&
+                // amplitude term e^2 must be negligible; a phase that is not
+                // finite is not masked by a zero amplitude
+                const bool series_ok = fabs(cyc0) <= 1.0 && e * e * e * rc * g.inv_lambda < 16 * 2e-7 && e * e < 1e-7 &&
                                        nmax * 0.5 * g.inv_lambda / rc <= MAX_CYC;
                 if (!series_ok) {
                     cls = CLS_EXACT;
@@ -604,7 +606,7 @@ __device__ __attribute__((always_inline)) inline void exact_tile(ExactSmem& sm, 
         if (tid < XCH && p < p_end) {
             b = s.box[p];
             if (b.x < cx1 && b.y > x0 && b.z < ry1 && b.w > y0)
-                ex = left_pair<double>(g, s.px[p], s.py[p], s.pz[p], s.kamp[p], b, x0, y0);
+                ex = left_pair<double>(g, s.px[p], s.py[p], s.pz[p], s.cyc0[p], s.kamp[p], b, x0, y0);
         }
         // listed in point order
         const unsigned long long m = __ballot(ex);
@@ -761,7 +763,7 @@ __device__ __attribute__((always_inline)) inline void line_strip(LineSmem& sm, c
                 const double px = s.px[p], py = s.py[p], z = s.pz[p];
                 int4 ib;
                 if (dgemm::inner_box(g, px, py, z, b, ib) &&
-                    !((left & dgemm::LEFT_PAIRS) && left_pair<T>(g, px, py, z, s.kamp[p], b, x0, y0))) {
+                    !((left & dgemm::LEFT_PAIRS) && left_pair<T>(g, px, py, z, s.cyc0[p], s.kamp[p], b, x0, y0))) {
                     m = dgemm::edge_lines(b, ib, x0, x1, y0, y1);
                     cut = (unsigned)(ib.x - b.x) | (unsigned)(b.y - ib.y) << 1;
                 }

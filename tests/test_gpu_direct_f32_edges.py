@@ -73,3 +73,27 @@ def test_amplitudes(ctx, amp, diff, mode, tol):
     v = synth.random_cloud(6600, 40, 1.5e-3, (0.02, 0.03)).copy()
     v["color"][17] = amp
     check(ctx, v, (400, 300), (8e-6, 8e-6), diff, mode, tol)
+
+
+# a phase that is not finite: NaN at the pixels of the point's mask (of the whole
+# hologram where the mask covers it), as in the probe, and only there; few points
+# on a large hologram take the per-pixel kernel in RS FP32, the others the matrix
+# products
+@pytest.mark.parametrize("mode,tol", [(FP64, 1e-11), (FP32, 1e-5)])
+@pytest.mark.parametrize("diff", [0, 1])
+@pytest.mark.parametrize("phase", [float("nan"), float("inf"), -float("inf")])
+@pytest.mark.parametrize("pn,n,z", [((400, 300), 40, (0.02, 0.03)), ((900, 500), 40, (0.02, 0.03)),
+                                    ((700, 400), 700, (0.1, 0.2)), ((700, 400), 700, (0.05, 0.06))])
+def test_phases_not_finite(ctx, pn, n, z, phase, diff, mode, tol):
+    v = synth.random_cloud(6650, n, 1.5e-3, z, complex_amplitude=True).copy()
+    v["phase"][17] = phase
+    pp = (8e-6, 8e-6)
+    got = capi.generate(ctx, v, pn, pp, [LAM], diff, mode, use_phase=True)[0].ravel()
+    dv = ctx.to_device(v)
+    try:
+        want = ctx.probe_f64(dv, len(v), capi.params(pn, pp, LAM, use_phase=True), diff, np.arange(pn[0] * pn[1]))
+    finally:
+        dv.free()
+    finite = np.isfinite(want)
+    assert not finite.all() and np.array_equal(np.isfinite(got), finite)
+    assert np.linalg.norm(got[finite] - want[finite]) <= tol * np.linalg.norm(want[finite])
