@@ -37,6 +37,7 @@
 //    layout) is read-modify-written once per pixel and kernel.
 #include <climits>
 
+#include "line_entry.h"
 #include "ohx_internal.h"
 
 namespace ohx {
@@ -706,7 +707,7 @@ __global__ __launch_bounds__(NT) void k_pc_rest(Geometry g, PointSoA s, double2*
 constexpr int LINE_ROWS = 8;
 struct LineSmem {
     double2 acc[LINE_ROWS][64];
-    int queue[128];   // points whose column lines wait; bit 0: last column
+    int64_t queue[128];   // column lines that wait (line_entry; points from p_begin)
 };
 
 template <typename T>
@@ -737,10 +738,10 @@ __device__ __attribute__((always_inline)) inline void line_strip(LineSmem& sm, c
         double re = 0.0, im = 0.0;
         int c = 0;
         if (i < n) {
-            const int e = sm.queue[i];
-            const int4 b = s.box[p_begin + (e >> 1)];
-            c = (e & 1) ? b.y - 1 : b.x;
-            if (row >= b.z && row < b.w) term(p_begin + (e >> 1), pix_x(g, c), pix_y(g, row), re, im);
+            const int64_t e = sm.queue[i], p = p_begin + line_point(e);
+            const int4 b = s.box[p];
+            c = line_side(e) ? b.y - 1 : b.x;
+            if (row >= b.z && row < b.w) term(p, pix_x(g, c), pix_y(g, row), re, im);
         }
         for (int k = 0; k < n; ++k) {   // line by line: the order of the sums is the queue's
             if (i == k) {
@@ -795,7 +796,7 @@ __device__ __attribute__((always_inline)) inline void line_strip(LineSmem& sm, c
             if ((m >> side) & 1u)
                 sm.queue[waiting + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(has >> 32),
                                                                   __builtin_amdgcn_mbcnt_lo((unsigned)has, 0u))] =
-                    (int)(p - p_begin) * 2 + side;
+                    line_entry(p - p_begin, side);
             waiting += __popcll(has);
             any |= has != 0;
             wave_sync();
@@ -803,7 +804,7 @@ __device__ __attribute__((always_inline)) inline void line_strip(LineSmem& sm, c
                 columns(8);
                 waiting -= 8;
                 // up to 63 are left: move them to the front
-                const int e = lane < waiting ? sm.queue[lane + 8] : 0;
+                const int64_t e = lane < waiting ? sm.queue[lane + 8] : 0;
                 wave_sync();
                 if (lane < waiting) sm.queue[lane] = e;
                 wave_sync();
