@@ -5,10 +5,8 @@
 // and pixel.  The generation of the 192 factors per point and 128 x 64 tile
 // comes on top: FP64 MFMA and any VALU instruction do not issue side by side
 // (measured: a wave of MFMAs and one of FMAs on a SIMD take the sum of their
-// times), so it is kept short: Fresnel phases are quadratic along a thread's
-// rows and columns and advance by complex rotations.
-// Fresnel, 20k points at 3840x2160: 48.6 -> 22.8 ms (19.4 of them products;
-// with a sine and cosine per factor 26.8); RS, 10k points at 1920x1080: 19.1 ->
+// times).
+// Fresnel, 20k points at 3840x2160: 48.6 -> 23.7 ms (19.4 of them products); RS, 10k points at 1920x1080: 19.1 ->
 // 11.2 ms.  The scalar form read one row factor from LDS per 4 FMAs and wave
 // (Fresnel) and spent 23 FP64 instructions per pair (RS).  128 x 64 pixels is
 // the largest tile whose sums fit 256 registers with two workgroups per CU.
@@ -24,7 +22,7 @@ constexpr int NLIST = 128;              // listed points of a chunk, each rank's
 struct Smem64 {
     double v[64][ROWD], u[GW][ROWD];    // slot s, point i of it: re at s * 4 + i, im at s * 4 + 2 + i
     double2 tab[NTAB];                  // (cos, sin)(2 pi i / NTAB)
-    double c[9][NLIST];
+    double c[6][NLIST];
     unsigned box[NLIST];                // rows [b0, b1), columns [b2, b3) of the tile, byte k = bk
     int cnt[2][2][Kind<double>::RMAX + 1];   // [chunk parity][wave][rank]
     int left[2];                        // pairs, box edge lines of pairs left to the per-pixel kernel
@@ -34,9 +32,11 @@ struct Smem64 {
 __device__ inline void cis(double t, const double2* tab, double& c, double& s) { sincos2pi(t - floor(t), tab, s, c); }
 
 // Fresnel factors of one batch (listed points j0 .. j0 + n - 1): thread = one
-// point and every 16th column and row; the factor advances by the rotation
-// e^{j 2pi difference}, the difference by the point's second difference (two
-// complex products per factor, at most 7 steps).
+// point and every 16th column and row, each factor from its own phase.  (Factors
+// advanced by rotations, 20k points at 3840x2160, 22.9 ms against 23.7: but their
+// angles are rounded at the size of a step's phase, tens of cycles for a point
+// near the hologram, which left the field off by 1.5e-13 to 3.5e-13 at all
+// depths from 1 mm; by 6e-16 (1 mm) to 1.6e-13 (0.3 m) with phases of their own.)
 __device__ inline void gen_fresnel(Smem64& sm, const Geometry& g, int j0, int n, int tid, int x0, int y0)
 {
     constexpr int PB = 2 * SLOTS, NG = NT / PB;
@@ -48,35 +48,20 @@ __device__ inline void gen_fresnel(Smem64& sm, const Geometry& g, int j0, int n,
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
         const bool rows = side == 1;
-        const int N = (rows ? 64 : GW) / NG;
         const unsigned lo = (rows ? box : box >> 16) & 255u, hi = (rows ? box >> 8 : box >> 24) & 255u;
-        const double st = rows ? -(NG * g.pp_y) : NG * g.pp_x;
-        const double d = rows ? pix_y(g, y0 + grp) - sm.c[F_PY][j] : pix_x(g, x0 + grp) - sm.c[F_PX][j];
-        double c, s, dc, ds;
-        cis(fresnel_cycles(q, d) + (rows ? sm.c[F_CYC][j] : 0.0), sm.tab, c, s);
-        cis((q * st) * fma(2.0, d, st), sm.tab, dc, ds);
-        const double wc = sm.c[rows ? F_WYR : F_WXR][j], ws = sm.c[rows ? F_WYI : F_WXI][j];
-        if (rows) {
-            c *= sm.c[F_AMP][j];
-            s *= sm.c[F_AMP][j];
-        }
+        const double at0 = sm.c[rows ? F_PY : F_PX][j], cyc = sm.c[F_CYC][j], amp = rows ? sm.c[F_AMP][j] : 1.0;
         double* dst = (rows ? sm.v[grp] : sm.u[grp]) + at;
 #pragma unroll
-        for (int i = 0; i < N; ++i) {
+        for (int i = 0; i < (rows ? 64 : GW) / NG; ++i) {
             const unsigned k = grp + NG * i;
-            const bool in = k >= lo && k < hi;
-            dst[NG * i * ROWD] = in ? c : 0.0;
-            dst[NG * i * ROWD + 2] = in ? s : 0.0;
-            if (i + 1 < N) {
-                const double c1 = fma(c, dc, -(s * ds)), s1 = fma(c, ds, s * dc);
-                c = c1;
-                s = s1;
-            }
-            if (i + 2 < N) {
-                const double c1 = fma(dc, wc, -(ds * ws)), s1 = fma(dc, ws, ds * wc);
-                dc = c1;
-                ds = s1;
-            }
+            const double d = (rows ? pix_y(g, y0 + k) : pix_x(g, x0 + k)) - at0;
+            // mod 1 of the unrounded last product
+            const double qd = q * d, t = fma(qd, d, -floor(qd * d));
+            double c, s;
+            sincos2pi(rows ? t + cyc : t, sm.tab, s, c);
+            const double a = k >= lo && k < hi ? amp : 0.0;
+            dst[NG * i * ROWD] = a * c;
+            dst[NG * i * ROWD + 2] = a * s;
         }
     }
 }
@@ -172,7 +157,7 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
 {
     constexpr int UN = Kind<double>::UNIT, GH = Kind<double>::GH;
     constexpr int RMIN = DIFF == OHX_DIFF_RS ? 2 : 1, RMAX = DIFF == OHX_DIFF_RS ? Kind<double>::RMAX : 1;
-    constexpr int NC = DIFF == OHX_DIFF_RS ? 6 : 9;
+    constexpr int NC = DIFF == OHX_DIFF_RS ? 6 : 5;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int x0 = (tile % tiles_x) * GW, y0 = (tile / tiles_x) * GH;
     const int cx1 = min(x0 + GW, g.pn_x), ry1 = min(y0 + GH, g.pn_y);
@@ -215,12 +200,6 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
                 else if (DIFF == OHX_DIFF_RS && edge_lines(b, ib, x0, cx1, y0, ry1)) sm.left[1] = 1;
                 bb = box_bits(ib, x0, y0);
                 point_constants<DIFF>(g, s, p, px, py, z, q, pix_x(g, x0 + GW / 2), pix_y(g, y0 + GH / 2), cc);
-                if constexpr (DIFF == OHX_DIFF_FRESNEL) {
-                    constexpr int NG = NT / (2 * SLOTS);
-                    const double sx = NG * g.pp_x, sy = NG * g.pp_y;
-                    cis(q * (2.0 * sx * sx), sm.tab, cc[F_WXR], cc[F_WXI]);
-                    cis(q * (2.0 * sy * sy), sm.tab, cc[F_WYR], cc[F_WYI]);
-                }
             }
         }
         // counts per rank of waves 0 and 1, which hold the chunk's points (by

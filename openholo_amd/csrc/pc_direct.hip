@@ -201,7 +201,7 @@ __device__ inline void exact_term(double dx, double dy, double z, double cyc0, d
 // FP32 factors and FP32 sums over a chunk, folded into FP64).
 constexpr int NTAB = 256;  // angles of the FP64 sin/cos table
 
-// sin and cos of 2 pi t, t in [0, 1], in FP64: the nearest table angle
+// sin and cos of 2 pi t, t in [0, 2], in FP64: the nearest table angle
 // 2 pi i / NTAB plus Taylor series of the remainder |x| <= pi / NTAB
 // (dropped terms below 2e-20), combined by angle addition; about 17 FP64
 // instructions and one LDS read against ~40 for sincospi.

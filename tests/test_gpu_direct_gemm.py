@@ -59,3 +59,13 @@ def test_tile_and_point_remainders(ctx, pn, n, diff, mode, tol):
 def test_depths(ctx, z, diff, mode, tol):
     v = synth.random_cloud(6200 + int(1e3 * z[0]), 150, 2e-3, z)
     check(ctx, v, (420, 300), (8e-6, 8e-6), diff, mode, tol)
+
+
+# Fresnel near the hologram, where phases are small: the FP64 sums and the probe
+# round phases of at most lambda z / (4 pitch^2) cycles (both axes at the box
+# corner) to half a unit in the last place, a few times each
+@pytest.mark.parametrize("pp", [8e-6, 3.74e-6])
+@pytest.mark.parametrize("z", [1e-3, 3e-3, 1e-2])
+def test_fresnel_fp64_phase_rounding(ctx, z, pp):
+    v = synth.random_cloud(6250, 200, 200 * pp, (0.9 * z, z), complex_amplitude=True)
+    check(ctx, v, (700, 500), (pp, pp), 1, FP64, 8 * np.pi * (LAM * z / (4 * pp * pp) + 1) * 2.0**-53, use_phase=True)
