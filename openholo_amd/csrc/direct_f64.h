@@ -6,10 +6,11 @@
 // comes on top: FP64 MFMA and any VALU instruction do not issue side by side
 // (measured: a wave of MFMAs and one of FMAs on a SIMD take the sum of their
 // times).
-// Fresnel, 20k points at 3840x2160: 48.6 -> 23.7 ms (19.4 of them products); RS, 10k points at 1920x1080: 19.1 ->
-// 11.2 ms.  The scalar form read one row factor from LDS per 4 FMAs and wave
-// (Fresnel) and spent 23 FP64 instructions per pair (RS).  128 x 64 pixels is
-// the largest tile whose sums fit 256 registers with two workgroups per CU.
+// Fresnel, 20k points at 3840x2160: 48.6 -> 23.7 ms (19.4 of them products); RS,
+// 10k points at 1920x1080: 19.1 -> 11.2 ms.  The scalar form read one row factor
+// from LDS per 4 FMAs and wave (Fresnel) and spent 23 FP64 instructions per pair
+// (RS).  128 x 64 pixels is the largest tile whose sums fit 256 registers with two
+// workgroups per CU.
 #pragma once
 
 namespace dgemm {
@@ -27,9 +28,6 @@ struct Smem64 {
     int cnt[2][2][Kind<double>::RMAX + 1];   // [chunk parity][wave][rank]
     int left[2];                        // pairs, box edge lines of pairs left to the per-pixel kernel
 };
-
-// (cos, sin)(2 pi t)
-__device__ inline void cis(double t, const double2* tab, double& c, double& s) { sincos2pi(t - floor(t), tab, s, c); }
 
 // Fresnel factors of one batch (listed points j0 .. j0 + n - 1): thread = one
 // point and every 16th column and row, each factor from its own phase.  (Factors
@@ -81,7 +79,7 @@ __device__ inline void gen_rs(Smem64& sm, const Geometry& g, int j0, int m, int 
         const unsigned lo = (rows ? box : box >> 16) & 255u, hi = (rows ? box >> 8 : box >> 24) & 255u;
         const double g2 = sm.c[rows ? R_G2Y : R_G2X][j];
         const double wc = rows ? pix_y(g, y0 + 32) : pix_x(g, x0 + GW / 2);
-        const double cyc = rows ? sm.c[R_CYC][j] : 0.0, amp = rows ? sm.c[R_AMP][j] : 1.0;
+        const double cyc = sm.c[R_CYC][j], amp = rows ? sm.c[R_AMP][j] : 1.0;
         const double ir = sm.c[R_IR][j], rho = sm.c[R_RHO][j];
 #pragma unroll 1
         for (int k0 = grp; k0 < (rows ? 64 : GW); k0 += NG) {
@@ -91,8 +89,10 @@ __device__ inline void gen_rs(Smem64& sm, const Geometry& g, int j0, int m, int 
             const double t =
                 e * fma(e, fma(e, fma(e, fma(e, fma(e, -21.0 / 1024.0, 7.0 / 256.0), -5.0 / 128.0), 1.0 / 16.0), -0.125),
                         0.5);
+            // mod 1 of the unrounded product
+            const double ph = fma(rho, t, -floor(rho * t));
             double c, s;
-            cis(fma(rho, t, cyc), sm.tab, c, s);
+            sincos2pi(rows ? ph + cyc : ph, sm.tab, s, c);
             double a = amp * pure_amp<double>(e);
             a = ((unsigned)k0 >= lo && (unsigned)k0 < hi) ? a : 0.0;
             double* dst = (rows ? sm.v[k0] : sm.u[k0]) + at;

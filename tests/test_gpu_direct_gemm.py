@@ -69,3 +69,27 @@ def test_depths(ctx, z, diff, mode, tol):
 def test_fresnel_fp64_phase_rounding(ctx, z, pp):
     v = synth.random_cloud(6250, 200, 200 * pp, (0.9 * z, z), complex_amplitude=True)
     check(ctx, v, (700, 500), (pp, pp), 1, FP64, 8 * np.pi * (LAM * z / (4 * pp * pp) + 1) * 2.0**-53, use_phase=True)
+
+
+# one RS point at a time, where the terms dropped beside the last power of the
+# expansion weigh most (6th rank, the largest tiles that the product takes), and at
+# depths that take all ranks: no pixel is off by more than the tolerance of the
+# expansion, 2e-13, and the rounding of the phases
+@pytest.mark.parametrize("x,y,z", [(8e-5, 8.1e-4, 0.0252), (-4e-4, -8.1e-4, 0.0207), (3.5e-4, 8.8e-4, 0.0286),
+                                   (-1e-4, 6.5e-4, 0.0222), (5.2e-4, -9e-4, 0.0246), (0.0, 0.0, 0.06),
+                                   (1e-3, -1e-3, 0.12), (2e-3, 1e-3, 0.3), (-1e-3, 2e-3, 0.6)])
+def test_rs_fp64_single_points(ctx, x, y, z):
+    v = synth.random_cloud(6260, 1, 1e-3, (0.1, 0.2)).copy()
+    v["pos"][0] = x, y, z
+    pn, pp = (700, 500), (8e-6, 8e-6)
+    got = capi.generate(ctx, v, pn, pp, [LAM], 0, FP64)[0].ravel()
+    dv = ctx.to_device(v)
+    try:
+        want = ctx.probe_f64(dv, 1, capi.params(pn, pp, LAM), 0, np.arange(pn[0] * pn[1]))
+    finally:
+        dv.free()
+    inside = want != 0
+    assert np.array_equal(got != 0, inside)
+    err = float(np.max(np.abs(got - want)[inside] / np.abs(want[inside])))
+    print(f"z {z}: {err:.2e}")
+    assert err < 2e-13 + 8 * np.pi * (LAM * z / (4 * pp[0] * pp[1]) + 1) * 2.0**-53
