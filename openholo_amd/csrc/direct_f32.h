@@ -563,7 +563,7 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem32<DIFF>&
                           acc.d[cb][1][i]);
     }
     if constexpr (DIFF == OHX_DIFF_FRESNEL) {
-        if (sm.left[0]) add_left<float>(g, s, p_begin, p_end, field, part, x0, y0);
+        if (sm.left[0]) add_left<float>((int*)&sm.f, g, s, p_begin, p_end, field, part, x0, y0);
     }
     return (unsigned)(sm.left[0] | sm.left[1] << 1);
 }

@@ -267,7 +267,7 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
                               acc.a[rb][cb][0][i], acc.a[rb][cb][1][i]);
     }
     if constexpr (DIFF == OHX_DIFF_FRESNEL) {
-        if (sm.left[0]) add_left<double>(g, s, p_begin, p_end, field, part, x0, y0);
+        if (sm.left[0]) add_left<double>((int*)&sm.v, g, s, p_begin, p_end, field, part, x0, y0);
     }
     return (unsigned)(sm.left[0] | sm.left[1] << 1);
 }

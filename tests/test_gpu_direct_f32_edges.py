@@ -97,3 +97,16 @@ def test_phases_not_finite(ctx, pn, n, z, phase, diff, mode, tol):
     finite = np.isfinite(want)
     assert not finite.all() and np.array_equal(np.isfinite(got), finite)
     assert np.linalg.norm(got[finite] - want[finite]) <= tol * np.linalg.norm(want[finite])
+
+
+# clouds that Fresnel in FP32 leaves to the FP64 terms altogether (amplitudes below
+# the products' range), around the points tested at a time and with some that the
+# products take between them: FP64 accuracy
+@pytest.mark.parametrize("n", [1, 511, 512, 513, 1100])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_fresnel_fp32_left_points(ctx, n, mixed):
+    v = synth.random_cloud(6680 + n, n, 1.5e-3, (0.02, 0.03)).copy()
+    v["color"] *= 1e-38
+    if mixed:
+        v["color"][n // 3:n // 2] = 0.0
+    check(ctx, v, (300, 200), (8e-6, 8e-6), 1, FP32, 1e-11)
