@@ -110,3 +110,16 @@ def test_fresnel_fp32_left_points(ctx, n, mixed):
     if mixed:
         v["color"][n // 3:n // 2] = 0.0
     check(ctx, v, (300, 200), (8e-6, 8e-6), 1, FP32, 1e-11)
+
+
+# faint clouds: their products keep every part of a factor down to amplitudes (in
+# the field) of 1e-30
+@pytest.mark.parametrize("diff", [0, 1])
+@pytest.mark.parametrize("scale", [1e-12, 1e-25, 1e-30, 1e-35, 1e-36])
+def test_fp32_faint_clouds(ctx, scale, diff):
+    v = synth.random_cloud(6690, 300, 1.5e-3, (0.25, 0.3)).copy()
+    ref = capi.generate(ctx, v, (300, 200), (8e-6, 8e-6), [LAM], diff, FP32)[0]
+    v["color"] *= scale
+    got = capi.generate(ctx, v, (300, 200), (8e-6, 8e-6), [LAM], diff, FP32)[0] / scale
+    # both round to FP32
+    assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref)
