@@ -62,6 +62,11 @@ int geometry_from_params(ohx_ctx* ctx, const ohx_pc_params* p, uint32_t diff, Ge
     const double sqrtX = std::sqrt(1 - (tx * tx)), sqrtY = std::sqrt(1 - (ty * ty));
     g->hx_coef = tx / sqrtX;
     g->hy_coef = ty / sqrtY;
+    // such pixels are centred within half_box + (34 + |offset|, 18 + |offset|) pitches
+    // of the point and q half_box is 1 / (4 pitch), so q (2 u d + u^2 + 2 v d' + v^2),
+    // u = 32 and v = 16 pitches, is at most 24 + q times the sum below
+    const double ox = std::fabs((double)p->offset_x), oy = std::fabs((double)p->offset_y);
+    g->q_near = 40.0 / ((3200.0 + 64.0 * ox) * p->pp_x * p->pp_x + (832.0 + 32.0 * oy) * p->pp_y * p->pp_y);
     for (int i = 0; i < 3; ++i) g->scale[i] = p->scale[i];
     g->distance = p->distance;
     g->channel = p->channel;

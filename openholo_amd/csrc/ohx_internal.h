@@ -84,6 +84,9 @@ struct Geometry {
     double x0, y0;       // -ss_x/2, -ss_y/2
     double lambda, inv_lambda;
     double hx_coef, hy_coef;  // RS: tx/sqrt(1-tx^2); Fresnel: unused
+    // Fresnel: above this PointSoA::q a phase may run over more than 64 cycles on 64 x
+    // 32 pixels that meet the point's box
+    double q_near;
     double scale[3];
     double distance;
     int32_t channel, use_phase;

@@ -123,3 +123,12 @@ def test_fp32_faint_clouds(ctx, scale, diff):
     got = capi.generate(ctx, v, (300, 200), (8e-6, 8e-6), [LAM], diff, FP32)[0] / scale
     # both round to FP32
     assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref)
+
+
+# Fresnel points so near that a phase runs over more than 64 cycles on 64 x 32
+# pixels (boxes of at most 25 pixels here): FP64 terms in FP32 mode too
+@pytest.mark.parametrize("pn,n,pp,z", [((300, 200), 300, 8e-6, (1e-3, 3e-3)), ((130, 129), 2000, 8e-6, (0.5e-3, 2e-3)),
+                                       ((700, 500), 900, 3.74e-6, (0.2e-3, 0.6e-3))])
+def test_fresnel_fp32_nearest_points(ctx, pn, n, pp, z):
+    v = synth.random_cloud(6695 + n, n, 0.6 * pn[1] * pp, z, complex_amplitude=True)
+    check(ctx, v, pn, (pp, pp), 1, FP32, 1e-11, use_phase=True)
