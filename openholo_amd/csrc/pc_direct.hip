@@ -579,44 +579,67 @@ __device__ inline void split_item(const Geometry& g, const PointSoA& s, const Sp
 
 // ---------------------------------------------------------------------------
 // The pairs that the matrix products leave (direct_gemm.h), pixel by pixel:
-// every term in FP64 under the reference's mask, on one 64 x 32 tile.
-constexpr int XCH = 128;   // points per chunk
-struct ExactSmem {
-    double d[5][XCH];      // px, py, z, cyc0, kamp
-    int4 box[XCH];
-    int cnt[2];
+// every term in FP64 under the reference's mask, 64 columns x 8 rows a wave, a lane
+// per column.  RG waves take the rows of a tile; near the hologram all points may
+// be left, and where tiles are few, SHARES waves share the listed points of a row
+// group, and their sums are added in a fixed order.  SHARES = 16 where the hologram
+// has fewer tiles of 64 x 32 than two a CU (10k points at 320x180, z 5 to 20 mm: 3.4
+// ms against 17.9 with one share; 3k at 640x360: 0.45 against 1.8), else 1 and RG =
+// 4 (20k at 1920x1080, 1 to 4 mm: 0.76 ms against 1.16 with 16: more tiles to list,
+// and sums to add).
+constexpr int XROWS = RPT;
+template <int SHARES, int RG>
+union ExactSmem {
+    struct {
+        double d[5][64 * SHARES * RG];   // px, py, z, cyc0, kamp of the listed points of a chunk
+        int4 box[64 * SHARES * RG];
+        int cnt[SHARES * RG];
+    };
+    double2 sum[SHARES > 1 ? SHARES / 2 * RG : 1][XROWS][64];
 };
+inline __host__ __device__ bool few_tiles(const Geometry& g)
+{
+    return (int64_t)((g.pn_x + TW - 1) / TW) * ((g.pn_y + TH - 1) / TH) < 512;
+}
 
-__device__ __attribute__((always_inline)) inline void exact_tile(ExactSmem& sm, const Geometry& g, const PointSoA& s,
-                                                                 int64_t p_begin, int64_t p_end,
+template <int SHARES, int RG>
+__device__ __attribute__((always_inline)) inline void exact_tile(ExactSmem<SHARES, RG>& sm, const Geometry& g,
+                                                                 const PointSoA& s, int64_t p_begin, int64_t p_end,
                                                                  double2* __restrict__ field, int x0, int y0)
 {
-    const int tid = threadIdx.x & (NT - 1), lane = tid & 63, wave = tid >> 6;
-    const int cx1 = min(x0 + TW, g.pn_x), ry1 = min(y0 + TH, g.pn_y);
-    const int col = x0 + lane, rowb = y0 + wave * RPT;
+    constexpr int W = SHARES * RG, N = 64 * W;   // waves; threads, points per chunk
+    const int tid = threadIdx.x & (N - 1), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int share = wave % SHARES, rg = wave / SHARES;
+    const int cx1 = min(x0 + 64, g.pn_x), ry1 = min(y0 + RG * XROWS, g.pn_y);
+    const int col = x0 + lane, row0 = y0 + rg * XROWS;
     const double xxx = pix_x(g, col);
-    double accr[RPT], acci[RPT];
+    double accr[XROWS], acci[XROWS];
 #pragma unroll
-    for (int k = 0; k < RPT; ++k) accr[k] = acci[k] = 0.0;
+    for (int k = 0; k < XROWS; ++k) accr[k] = acci[k] = 0.0;
     bool any = false;   // uniform: some pair on this tile
 
-    for (int64_t base = p_begin; base < p_end; base += XCH) {
+    for (int64_t base = p_begin; base < p_end; base += N) {
         bool ex = false;
         const int64_t p = base + tid;
         int4 b = make_int4(0, 0, 0, 0);
-        if (tid < XCH && p < p_end) {
+        if (p < p_end) {
             b = s.box[p];
             if (b.x < cx1 && b.y > x0 && b.z < ry1 && b.w > y0)
                 ex = left_pair<double>(g, s.px[p], s.py[p], s.pz[p], s.cyc0[p], s.kamp[p], b, x0, y0);
         }
         // listed in point order
         const unsigned long long m = __ballot(ex);
-        if (lane == 0 && wave < 2) sm.cnt[wave] = __popcll(m);
+        if (lane == 0) sm.cnt[wave] = __popcll(m);
         __syncthreads();
-        const int n0 = sm.cnt[0], n = __builtin_amdgcn_readfirstlane(n0 + sm.cnt[1]);
+        int n = 0, at = 0;
+        for (int w = 0; w < W; ++w) {
+            if (w == wave) at = n;
+            n += sm.cnt[w];
+        }
+        n = __builtin_amdgcn_readfirstlane(n);
         if (ex) {
-            const int j = (wave == 1 ? n0 : 0) + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                                           __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+            const int j =
+                at + __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
             sm.d[0][j] = s.px[p];
             sm.d[1][j] = s.py[p];
             sm.d[2][j] = s.pz[p];
@@ -626,15 +649,15 @@ __device__ __attribute__((always_inline)) inline void exact_tile(ExactSmem& sm, 
         }
         __syncthreads();
         any |= n > 0;
-        for (int j = 0; j < n; ++j) {
+        for (int j = share; j < n; j += SHARES) {
             const int4 bb = sm.box[j];
             const double qpx = sm.d[0][j], qpy = sm.d[1][j], qz = sm.d[2][j];
             const double qc = sm.d[3][j], qk = sm.d[4][j];
             const double zz = qz * qz;
             const bool colin = col >= bb.x && col < bb.y;
 #pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                const int row = rowb + k;
+            for (int k = 0; k < XROWS; ++k) {
+                const int row = row0 + k;
                 const double yyy = pix_y(g, row);
                 bool in = colin && row >= bb.z && row < bb.w;
                 in = in && rs_range_ok(qpx, qpy, zz, g.hx_coef, g.hy_coef, xxx, yyy);
@@ -644,7 +667,26 @@ __device__ __attribute__((always_inline)) inline void exact_tile(ExactSmem& sm, 
         }
         __syncthreads();
     }
-    if (any) store_tile(g, field, col, rowb, accr, acci);
+    if (!any) return;
+    // the upper half of the shares to the lower one, until one is left
+#pragma unroll
+    for (int half = SHARES / 2; half > 0; half /= 2) {
+        if (share >= half && share < 2 * half) {
+#pragma unroll
+            for (int k = 0; k < XROWS; ++k) sm.sum[rg * (SHARES / 2) + share - half][k][lane] = make_double2(accr[k], acci[k]);
+        }
+        __syncthreads();
+        if (share < half) {
+#pragma unroll
+            for (int k = 0; k < XROWS; ++k) {
+                const double2 v = sm.sum[rg * (SHARES / 2) + share][k][lane];
+                accr[k] += v.x;
+                acci[k] += v.y;
+            }
+        }
+        __syncthreads();
+    }
+    if (share == 0) store_tile(g, field, col, row0, accr, acci);
 }
 
 // Workgroup = (tile, point split): blockIdx = split * tiles + tile; split 0
@@ -672,26 +714,30 @@ __global__ __launch_bounds__(dgemm::Kind<T>::NTH, 512 / dgemm::Kind<T>::NTH) voi
     if (DIFF == OHX_DIFF_RS && left && threadIdx.x == 0) atomicOr(&flags[tile & (TILE_FLAGS - 1)], left);
 }
 
-// RS: the pairs k_pc_gemm left, one workgroup per 64 x 32 tile; returns at once
-// where there are none.  In FP32 mode in FP32 where the series holds on the
-// smaller tile, otherwise in FP64.
-template <typename T>
-struct RestSmem {
-    using type = ExactSmem;
+// RS: the pairs k_pc_gemm left, one workgroup per 64 x 32 (FEW: 64 x 8) tile; returns at
+// once where there are none.  In FP32 mode in FP32 where the series holds on the smaller
+// tile, otherwise in FP64.
+template <typename T, bool FEW>
+struct Rest {
+    static constexpr int SHARES = FEW ? 16 : 1, RG = FEW ? 1 : WAVES;
+    static constexpr int THREADS = 64 * SHARES * RG, ROWS = XROWS * RG;
+    using Smem = ExactSmem<SHARES, RG>;
 };
 template <>
-struct RestSmem<float> {
-    using type = DirectSmem;
+struct Rest<float, false> {
+    static constexpr int THREADS = NT, ROWS = TH;
+    using Smem = DirectSmem;
 };
 
-template <typename T>
-__global__ __launch_bounds__(NT) void k_pc_rest(Geometry g, PointSoA s, double2* __restrict__ field, int tiles_x,
-                                                int gemm_tiles_x, const unsigned* __restrict__ flags, bool all)
+template <typename T, bool FEW>
+__global__ __launch_bounds__((Rest<T, FEW>::THREADS)) void k_pc_rest(Geometry g, PointSoA s, double2* __restrict__ field,
+                                                                   int tiles_x, int gemm_tiles_x,
+                                                                   const unsigned* __restrict__ flags, bool all)
 {
-    const int x0 = (blockIdx.x % tiles_x) * TW, y0 = (blockIdx.x / tiles_x) * TH;
+    const int x0 = (blockIdx.x % tiles_x) * TW, y0 = (blockIdx.x / tiles_x) * Rest<T, FEW>::ROWS;
     const int t = (y0 / dgemm::Kind<T>::GH) * gemm_tiles_x + x0 / dgemm::GW;
     if (!all && !(flags[t & (TILE_FLAGS - 1)] & dgemm::LEFT_PAIRS)) return;
-    __shared__ typename RestSmem<T>::type sm;
+    __shared__ typename Rest<T, FEW>::Smem sm;
     if constexpr (dgemm::Kind<T>::f64) exact_tile(sm, g, s, 0, s.n, field, x0, y0);
     else rest_tile(sm, g, s, 0, s.n, field, x0, y0, all);
 }
@@ -880,23 +926,27 @@ __global__ __launch_bounds__(dgemm::Kind<T>::NTH, 512 / dgemm::Kind<T>::NTH) voi
     }
 }
 
-// The pairs those left, 64 x 32 tiles of the jobs that have any
+// The pairs those left, 64 x 32 (FP64, few tiles: 64 x 8) tiles of the jobs that have any
 __global__ __launch_bounds__(NT) void k_pc_rest_jobs(const DirectJob* __restrict__ jobs,
                                                      const int* __restrict__ njobs_ptr)
 {
     __shared__ union {
         DirectSmem rs;
-        ExactSmem exact;
+        ExactSmem<1, WAVES> exact;
+        ExactSmem<WAVES, 1> shared;
     } sm;
     const int njobs = *njobs_ptr;
     int item = blockIdx.x;
     for (int k = 0; k < njobs; ++k) {
         const DirectJob& jb = jobs[k];
         if (!jb.per_pixel && !(jb.left & dgemm::LEFT_PAIRS)) continue;
-        const int xt = (jb.g.pn_x + TW - 1) / TW, tiles = xt * ((jb.g.pn_y + TH - 1) / TH);
+        const bool few = jb.fp64 && few_tiles(jb.g);
+        const int rows = few ? XROWS : TH, xt = (jb.g.pn_x + TW - 1) / TW;
+        const int tiles = xt * ((jb.g.pn_y + rows - 1) / rows);
         for (; item < tiles; item += gridDim.x) {
-            const int x0 = (item % xt) * TW, y0 = (item / xt) * TH;
-            if (jb.fp64) exact_tile(sm.exact, jb.g, jb.s, jb.p0, jb.p1, jb.field, x0, y0);
+            const int x0 = (item % xt) * TW, y0 = (item / xt) * rows;
+            if (few) exact_tile(sm.shared, jb.g, jb.s, jb.p0, jb.p1, jb.field, x0, y0);
+            else if (jb.fp64) exact_tile(sm.exact, jb.g, jb.s, jb.p0, jb.p1, jb.field, x0, y0);
             else rest_tile(sm.rs, jb.g, jb.s, jb.p0, jb.p1, jb.field, x0, y0, jb.per_pixel != 0);
             __syncthreads();   // LDS reuse across items
         }
@@ -1054,7 +1104,15 @@ static void launch_gemm(hipStream_t st, const Geometry& g, const PointSoA& soa, 
         const dim3 grid((unsigned)(xt * ((g.pn_y + TH - 1) / TH)));
         const unsigned* fl = flags;
         hipLaunchKernelGGL(k_pc_lines<T>, grid, dim3(NT), 0, st, g, soa, f, xt, tiles_x, fl);
-        hipLaunchKernelGGL(k_pc_rest<T>, grid, dim3(NT), 0, st, g, soa, f, xt, tiles_x, fl, false);
+        if constexpr (dgemm::Kind<T>::f64) {
+            if (few_tiles(g)) {
+                using R = Rest<T, true>;
+                hipLaunchKernelGGL((k_pc_rest<T, true>), dim3((unsigned)(xt * ((g.pn_y + R::ROWS - 1) / R::ROWS))),
+                                   dim3(R::THREADS), 0, st, g, soa, f, xt, tiles_x, fl, false);
+                return;
+            }
+        }
+        hipLaunchKernelGGL((k_pc_rest<T, false>), grid, dim3(NT), 0, st, g, soa, f, xt, tiles_x, fl, false);
     }
 }
 
@@ -1080,7 +1138,7 @@ int launch_direct_with(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, dou
     ctx->last.workgroups = fp64 ? (int64_t)tiles_x * ((g.pn_y + 15) / 16) : small_tiles;
     ctx->last.kernel_kind = fp64 ? 1 : 0;
     if (per_pixel) {
-        hipLaunchKernelGGL(k_pc_rest<float>, dim3((unsigned)small_tiles), dim3(NT), 0, ctx->stream, g, soa, f, xt, tiles_x,
+        hipLaunchKernelGGL((k_pc_rest<float, false>), dim3((unsigned)small_tiles), dim3(NT), 0, ctx->stream, g, soa, f, xt, tiles_x,
                            (const unsigned*)flags, true);
         return check_hip(ctx, hipGetLastError(), "k_pc_rest");
     }

@@ -93,3 +93,20 @@ def test_rs_fp64_single_points(ctx, x, y, z):
     err = float(np.max(np.abs(got - want)[inside] / np.abs(want[inside])))
     print(f"z {z}: {err:.2e}")
     assert err < 2e-13 + 8 * np.pi * (LAM * z / (4 * pp[0] * pp[1]) + 1) * 2.0**-53
+
+
+# RS points near the hologram, all left to the per-pixel FP64 terms: around the
+# points listed at a time (1024 or 256), the 64 x 8 tiles (64 x 32 from 512 of them) and the
+# shares of a tile (16, a server's job 4)
+@pytest.mark.parametrize("pn", [(64, 8), (65, 9), (70, 13), (130, 71), (1030, 961), (1030, 960)])
+@pytest.mark.parametrize("n", [1, 5, 17, 255, 257, 1023, 1025, 2100])
+def test_rs_fp64_left_points(ctx, pn, n):
+    pp = (8e-6, 8e-6)
+    v = synth.random_cloud(6270 + n, n, 0.6 * pn[1] * pp[1], (2e-3, 8e-3))
+    check(ctx, v, pn, pp, 0, FP64, 1e-11)
+    one = capi.generate(ctx, v, pn, pp, [LAM], 0, FP64)[0]
+    with capi.Server(0) as srv:
+        status, _, field, _ = srv.wait(srv.submit(v, capi.params(pn, pp, LAM), 0, FP64, want_field=True))
+    assert status == capi.OK
+    assert np.array_equal(field.reshape(one.shape) != 0, one != 0)
+    assert np.linalg.norm(field.reshape(one.shape) - one) <= 1e-11 * np.linalg.norm(one)
