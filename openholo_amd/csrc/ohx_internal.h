@@ -163,18 +163,6 @@ __device__ inline bool rs_mask_bit(const unsigned* __restrict__ row, int t)
     return (row[t >> 5] >> (t & 31)) & 1u;
 }
 
-// Points per FP32 partial sum for n points on a hologram: 240, or shorter ones, at
-// whose boundaries tiles are split, where 240 would leave CUs without work (256
-// workgroups of 240 points take 40 to 120 us; a fold costs 2 us of a group's
-// 10 to 100).
-inline int direct_chunk(const Geometry& g, int64_t n)
-{
-    const int64_t tiles = (int64_t)((g.pn_x + 127) / 128) * ((g.pn_y + 127) / 128);
-    int chunk = DIRECT_CHUNK;
-    while (chunk > (g.diff == OHX_DIFF_RS ? 1 : 2) * DIRECT_CELL && tiles * n < 256 * chunk) chunk /= 2;
-    return chunk;
-}
-
 // RS in FP32, whole cloud: the per-pixel kernel alone.  Its 64 x 32 tiles start
 // and end sooner than the matrix kernel's, and points near enough for rank 4 take
 // the same time per pair in either (300 points at 640 x 360: 78 us against 92;
@@ -242,6 +230,8 @@ int launch_direct_with(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, dou
 void noalloc_init(int device);
 int launch_fresnel_gemm(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, double* d_field, uint32_t mode);
 int direct_tiles(const Geometry& g, bool fp64, int* tiles_x);
+// points per FP32 partial sum for n points on a hologram (240, 120, 60 or 30)
+int direct_chunk(const Geometry& g, int64_t n);
 int wrp_generate(ohx_ctx* ctx, const void* d_vertices, int64_t n, const ohx_wrp_params* p, double* d_field,
                  double* d_wrp);
 void wrp_release(ohx_ctx* ctx);

@@ -1061,35 +1061,72 @@ static int resident_slots(ohx_ctx* ctx, const void* k, int threads)
     return per_cu * cus;
 }
 
-// Point splits of the matrix-product kernels: least time in units of 0.1 us, as
-// rounds of resident workgroups x (points per split at pc a point, plus `base` for
-// the tile's start and end), plus the write and read of each further partial
-// plane (32 B a pixel at ~4 TB/s) and one more launch.  Split boundaries are
-// multiples of `chunk` points, planes stay under 2 GiB.
+// Point splits of the matrix-product kernels by their modelled time, in units of 0.1
+// us: a point on a tile (FP32: with its share of a group's start and fold, 4 us for
+// Fresnel, 10 for RS), a tile's start and end, and each further partial plane
+// (written and read, 32 B a pixel at ~4 TB/s) with one more launch.  Split boundaries
+// are multiples of `chunk` points, planes stay under 2 GiB.
 constexpr int MAX_SPLITS = 64;
-static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, int chunk, double pc, double base)
+struct GemmCost {
+    double point, tile;
+};
+static GemmCost gemm_cost(bool rs, bool fp64, int chunk)
+{
+    if (fp64) return {rs ? 16.0 : 5.0, 60.0};
+    return rs ? GemmCost{4.4 + 100.0 / chunk, 200.0} : GemmCost{1.6 + 38.0 / chunk, 150.0};
+}
+
+// Time of `first` workgroups of c and then `tiles` of cl, each on the slot that is
+// free first.
+static double makespan(double first, double c, double tiles, double cl, double slots)
+{
+    const double full = std::floor(first / slots), rem = first - full * slots, open = slots - rem;
+    double t = std::ceil(tiles / open) * cl;   // on the slots that the last round of c leaves open
+    if (rem > 0.0) t = std::max(c, std::min(t, std::ceil((tiles + rem * c / cl) / slots) * cl));
+    return full * c + t;
+}
+
+static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, int chunk, GemmCost k, double* time)
 {
     int best = 1;
-    double best_t = 0.0;
     for (int S = 1; S <= MAX_SPLITS; ++S) {
-        if (S > 1 && (n < (int64_t)S * chunk || (double)(S - 1) * npx * 16.0 > 2.0 * (1ull << 30))) break;
+        if (S > 1 && (n < (int64_t)S * chunk || (double)(S - 1) * npx * 16.0 > 2.0 * (1ull << 30) ||
+                      tiles * (S - 1) > 8 * (int64_t)slots))
+            break;
         const int64_t per = S == 1 ? n : ((n + S - 1) / S + chunk - 1) / chunk * chunk, parts = (n + per - 1) / per;
-        const double rounds = std::ceil((double)tiles * parts / slots);
-        const double t = rounds * ((double)per * pc + base) + (S > 1 ? 40.0 + (parts - 1) * (npx * 8e-5) : 0.0);
-        if (S == 1 || t < best_t * 0.97) {
+        const double t = makespan((double)(tiles * (parts - 1)), per * k.point + k.tile, (double)tiles,
+                                  (n - (parts - 1) * per) * k.point + k.tile, slots) +
+                         (parts > 1 ? 40.0 + (parts - 1) * (npx * 8e-5) : 0.0);
+        // the first further plane by a tenth, for the model takes every box as whole
+        if (S == 1 || t < *time * (best == 1 ? 0.9 : 0.97)) {
             best = S;
-            best_t = t;
+            *time = t;
         }
     }
     return best;
 }
 
-// One point's time on one tile, in 0.1 us with every slot busy (RS at the usual
-// ranks 2 to 3 (FP32) and 3 to 4), FP32 with its share of a fold.
-static double gemm_point_cost(bool rs, bool fp64, int chunk)
+// 240, or shorter ones, at whose boundaries tiles are split, where 240 would leave
+// CUs without work (256 workgroups of 240 points), and shorter again where the model
+// finds them faster on the usual 256 CUs.  (Longer ones are faster for a few hundred
+// points on 1920x1080, by 14 us of 80 for 200 points, Fresnel; but an FP32 sum of 200
+// points is off by 3.1e-7, of 60 by 1.9e-7.)
+int direct_chunk(const Geometry& g, int64_t n)
 {
-    if (fp64) return rs ? 16.0 : 5.0;
-    return rs ? 4.0 + 25.0 / chunk : 1.6 + 15.0 / chunk;
+    const bool rs = g.diff == OHX_DIFF_RS;
+    int tx, best = DIRECT_CHUNK;
+    const int64_t tiles = direct_tiles(g, false, &tx), npx = (int64_t)g.pn_x * g.pn_y;
+    while (best > (rs ? 1 : 2) * DIRECT_CELL && tiles * n < 256 * best) best /= 2;
+    double best_t = 0.0;
+    for (int first = best, chunk = first; chunk >= DIRECT_CELL; chunk /= 2) {
+        double t;
+        gemm_point_splits(tiles, n, 256, npx, chunk, gemm_cost(rs, false, chunk), &t);
+        if (chunk == first || t < best_t * 0.97) {
+            best = chunk;
+            best_t = t;
+        }
+    }
+    return best;
 }
 
 // The matrix product, and for RS the per-pixel kernels for what it leaves.
@@ -1148,9 +1185,12 @@ int launch_direct_with(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, dou
                                   : (const void*)k_pc_gemm<OHX_DIFF_FRESNEL, float>);
     if (fp64) chunk = 32;
     int splits = 1;
-    if (allow_splits)
-        splits = gemm_point_splits(tiles, soa.n, resident_slots(ctx, kern, fp64 ? dgemm::Kind<double>::NTH : dgemm::Kind<float>::NTH),
-                                   npx, chunk, gemm_point_cost(rs, fp64, chunk), fp64 ? 60.0 : 100.0);
+    if (allow_splits) {
+        double t;
+        splits = gemm_point_splits(tiles, soa.n,
+                                   resident_slots(ctx, kern, fp64 ? dgemm::Kind<double>::NTH : dgemm::Kind<float>::NTH),
+                                   npx, chunk, gemm_cost(rs, fp64, chunk), &t);
+    }
     SplitArgs sa{(int)tiles, soa.n, nullptr, chunk};
     if (splits > 1) {
         // split boundaries on chunk boundaries: a split sums exactly as the
