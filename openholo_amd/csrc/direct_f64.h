@@ -6,7 +6,7 @@
 // comes on top: FP64 MFMA and any VALU instruction do not issue side by side
 // (measured: a wave of MFMAs and one of FMAs on a SIMD take the sum of their
 // times).
-// Fresnel, 20k points at 3840x2160: 48.6 -> 23.7 ms (19.4 of them products); RS,
+// Fresnel, 20k points at 3840x2160: 48.6 -> 23.5 ms (19.4 of them products); RS,
 // 10k points at 1920x1080: 19.1 -> 11.2 ms.  The scalar form read one row factor
 // from LDS per 4 FMAs and wave (Fresnel) and spent 23 FP64 instructions per pair
 // (RS).  128 x 64 pixels is the largest tile whose sums fit 256 registers with two
@@ -15,17 +15,20 @@
 
 namespace dgemm {
 
-constexpr int CH64 = 120;               // points per chunk
+// points per chunk: one per thread, listed in one go (120: clouds near the hologram,
+// where most points miss a tile, 20k at 1 to 4 mm on 1920x1080: Fresnel 361 us, now 247;
+// far ones 1 % slower)
+constexpr int CH64 = 240;
 constexpr int SLOTS = 8;                // K slots (two points of one rank) per batch
 constexpr int ROWD = SLOTS * 4 + 2;     // padded row of factors: 272 bytes, at which the operand reads do not conflict
-constexpr int NLIST = 128;              // listed points of a chunk, each rank's list padded to whole units
+constexpr int NLIST = 256;              // listed points of a chunk, each rank's list padded to whole units
 
 struct Smem64 {
     double v[64][ROWD], u[GW][ROWD];    // slot s, point i of it: re at s * 4 + i, im at s * 4 + 2 + i
     double2 tab[NTAB];                  // (cos, sin)(2 pi i / NTAB)
     double c[6][NLIST];
     unsigned box[NLIST];                // rows [b0, b1), columns [b2, b3) of the tile, byte k = bk
-    int cnt[2][2][Kind<double>::RMAX + 1];   // [chunk parity][wave][rank]
+    int cnt[2][NT / 64][Kind<double>::RMAX + 1];   // [chunk parity][wave][rank]
     int left[2];                        // pairs, box edge lines of pairs left to the per-pixel kernel
 };
 
@@ -202,8 +205,8 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
                 point_constants<DIFF>(g, s, p, px, py, z, q, pix_x(g, x0 + GW / 2), pix_y(g, y0 + GH / 2), cc);
             }
         }
-        // counts per rank of waves 0 and 1, which hold the chunk's points (by
-        // chunk parity: a slower wave may still read the last chunk's)
+        // counts per rank and wave (by chunk parity: a slower wave may still read the
+        // last chunk's)
         auto& cnt = sm.cnt[par];
         par ^= 1;
         int mine = 0;   // place among its wave's points of the same rank
@@ -212,15 +215,21 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
             const unsigned long long m = __ballot(rank == r);
             if (rank == r)
                 mine = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-            if (wave < 2 && lane == 0) cnt[wave][r] = __popcll(m);
+            if (lane == 0) cnt[wave][r] = __popcll(m);
         }
         __syncthreads();
         int beg = 0;
 #pragma unroll
         for (int r = RMIN; r <= RMAX; ++r) {
-            const int n0 = cnt[0][r], num = n0 + cnt[1][r], end = beg + (num + UN - 1) / UN * UN;
+            int num = 0, before = 0;
+#pragma unroll
+            for (int w = 0; w < NT / 64; ++w) {
+                before += w < wave ? cnt[w][r] : 0;
+                num += cnt[w][r];
+            }
+            const int end = beg + (num + UN - 1) / UN * UN;
             if (rank == r) {
-                const int j = beg + mine + (wave == 1 ? n0 : 0);
+                const int j = beg + mine + before;
 #pragma unroll
                 for (int i = 0; i < NC; ++i) sm.c[i][j] = cc[i];
                 sm.box[j] = bb;
@@ -240,7 +249,8 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
         beg = 0;
 #pragma unroll 1
         for (int r = RMIN; r <= RMAX; ++r) {
-            const int units = (__builtin_amdgcn_readfirstlane(cnt[0][r] + cnt[1][r]) + UN - 1) / UN;
+            const int units =
+                (__builtin_amdgcn_readfirstlane(cnt[0][r] + cnt[1][r] + cnt[2][r] + cnt[3][r]) + UN - 1) / UN;
             any |= units > 0;
             const int per = SLOTS / r;
 #pragma unroll 1

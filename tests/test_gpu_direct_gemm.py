@@ -110,3 +110,13 @@ def test_rs_fp64_left_points(ctx, pn, n):
     assert status == capi.OK
     assert np.array_equal(field.reshape(one.shape) != 0, one != 0)
     assert np.linalg.norm(field.reshape(one.shape) - one) <= 1e-11 * np.linalg.norm(one)
+
+
+# around the 240 points that the FP64 sums list at a time, over the depths of many
+# ranks (each rank's points padded in the list)
+@pytest.mark.parametrize("diff", [0, 1])
+@pytest.mark.parametrize("z", [(0.05, 0.06), (0.06, 1.5)])
+@pytest.mark.parametrize("n", [239, 240, 241, 255, 257, 481, 721])
+def test_fp64_listed_points(ctx, n, z, diff):
+    v = synth.random_cloud(6290 + n, n, 1.5e-3, z, complex_amplitude=True)
+    check(ctx, v, (300, 200), (8e-6, 8e-6), diff, FP64, 1e-11, use_phase=True)
