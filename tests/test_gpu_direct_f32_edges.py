@@ -132,3 +132,27 @@ def test_fp32_faint_clouds(ctx, scale, diff):
 def test_fresnel_fp32_nearest_points(ctx, pn, n, pp, z):
     v = synth.random_cloud(6695 + n, n, 0.6 * pn[1] * pp, z, complex_amplitude=True)
     check(ctx, v, pn, (pp, pp), 1, FP32, 1e-11, use_phase=True)
+
+
+# The FP32 sums hold FP32 factors in three BF16 parts.  What they round: phases to
+# 2^-25 cycles (2e-7 rad) and sines to about 1e-7 per factor, two factors a term, and
+# FP32 sums of up to 240 terms (up to 3e-7 of the sum); ranks cut at 4.5e-8: in all
+# below 1e-6.  A factor without its third part is off by up to 8e-6, a rank's factor
+# without its second by 3e-5 of the term.
+ROUNDING = 1e-6
+
+
+@pytest.mark.parametrize("pn,n,z", [((256, 256), 100, (0.1, 0.3)), ((256, 256), 2000, (0.1, 0.3)),
+                                    ((640, 500), 600, (0.3, 0.6)), ((500, 300), 300, (0.02, 0.04))])
+def test_fresnel_fp32_rounding(ctx, pn, n, z):
+    v = synth.random_cloud(6710 + n, n, 1e-3, z, complex_amplitude=True)
+    check(ctx, v, pn, (8e-6, 8e-6), 1, FP32, ROUNDING, use_phase=True)
+
+
+# depths at which points near the axis of 256 x 256 pixels take rank 2, 3 and 4
+# (theta = 1.83e-6 / z^3 at the far corner of a tile)
+@pytest.mark.parametrize("n", [100, 700, 2000])
+@pytest.mark.parametrize("z", [(0.3, 0.35), (0.08, 0.1), (0.042, 0.05)])
+def test_rs_fp32_rounding(ctx, n, z):
+    v = synth.random_cloud(6720 + n, n, 0.1e-3, z, complex_amplitude=True)
+    check(ctx, v, (256, 256), (8e-6, 8e-6), 0, FP32, ROUNDING, use_phase=True)
