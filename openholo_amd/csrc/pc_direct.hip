@@ -1108,20 +1108,23 @@ static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, i
 
 // 240, or shorter ones, at whose boundaries tiles are split, where 240 would leave
 // CUs without work (256 workgroups of 240 points), and shorter again where the model
-// finds them faster on the usual 256 CUs.  (Longer ones are faster for a few hundred
-// points on 1920x1080, by 14 us of 80 for 200 points, Fresnel; but an FP32 sum of 200
-// points is off by 3.1e-7, of 60 by 1.9e-7.)
+// finds a tenth in it on the usual 256 CUs (500 RS points at 1920x1080: 0.31 -> 0.27
+// ms; the serving engine and the no-allocation form sum alike but do not split, and
+// lose 8 %).  Longer ones are faster for a few hundred points on 1920x1080, by 14 us
+// of 80 for 200 points, Fresnel; but an FP32 sum of 200 points is off by 3.1e-7, of
+// 60 by 1.9e-7.
 int direct_chunk(const Geometry& g, int64_t n)
 {
     const bool rs = g.diff == OHX_DIFF_RS;
+    const int least = (rs ? 1 : 2) * DIRECT_CELL;
     int tx, best = DIRECT_CHUNK;
     const int64_t tiles = direct_tiles(g, false, &tx), npx = (int64_t)g.pn_x * g.pn_y;
-    while (best > (rs ? 1 : 2) * DIRECT_CELL && tiles * n < 256 * best) best /= 2;
+    while (best > least && tiles * n < 256 * best) best /= 2;
     double best_t = 0.0;
-    for (int first = best, chunk = first; chunk >= DIRECT_CELL; chunk /= 2) {
+    for (int first = best, chunk = first; chunk >= least; chunk /= 2) {
         double t;
         gemm_point_splits(tiles, n, 256, npx, chunk, gemm_cost(rs, false, chunk), &t);
-        if (chunk == first || t < best_t * 0.97) {
+        if (chunk == first || t < best_t * 0.9) {
             best = chunk;
             best_t = t;
         }
