@@ -252,10 +252,12 @@ int ohx_encode_normalize_u8(ohx_ctx* ctx, const double* const* d_field, int n_ch
 /* Shape of the last ohx_pc_diffract on ctx (for throughput accounting). */
 typedef struct ohx_launch_stats {
     int64_t pairs_nominal;   /* n_points * pn_x * pn_y                        */
-    int64_t workgroups;      /* direct sums: (tile, point split) items, in
-                                tiles of 64 x 32 (FP32) or 128 x 16 (FP64)
-                                pixels; matrix-core modes: workgroups of the
-                                kernel (Fresnel: of its unmasked instance,
+    int64_t workgroups;      /* direct sums: point splits times areas of 64 x 32
+                                (FP32) or 128 x 16 (FP64) pixels, a measure of
+                                the launch's division (the kernels' own tiles
+                                are 128 x 128 or 128 x 64); matrix-core
+                                modes: workgroups of the kernel (Fresnel: of
+                                its unmasked instance,
                                 which runs when every box covers the hologram) */
     int32_t kernel_kind;     /* 0 FP32 direct, 1 FP64 direct, 2 MFMA GEMM, 3 WRP */
     int32_t gemm_points;     /* RS with an MFMA mode: points that ran on the

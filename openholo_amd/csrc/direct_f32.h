@@ -11,15 +11,18 @@
 // by summing the negated terms of every second group).  With phases held as
 // 32-bit fractions of a cycle (Fresnel) or reduced in FP64 (RS), the field's
 // error against 64 bits is 3.5e-7 (Fresnel, 100k points, 3840x2160; 6.4e-7 with
-// scalar FP32 FMAs) and 3.9e-7 (RS, 20k points; 7.1e-7).
+// scalar FP32 FMAs) and 3.9e-7 (RS, 20k points; 7.1e-7); with 200 points, folded
+// every 60, 1.2e-7 to 2.4e-7 at depths to 1.2 m (2.9e-7 to 3.1e-6), or up to 7.4e-7
+// (2.1e-6) where the per-pixel kernel takes a part of the RS pairs.
 //
 // What bounds it: the matrix cores (48 flops per point and pixel for Fresnel, 72,
 // 96 and 144 for RS of ranks 2, 3 and 4) and the generation of 256 factors per
-// point and 128 x 128 tile on the VALU, which issues beside BF16 MFMAs (it does
-// not beside FP32 ones, whose 155 TFLOP/s this form beats).  So one workgroup of
-// 8 waves per CU, two per SIMD, and in each wave's stream the next batch's
-// generation alternates, slot by slot, with this batch's products
-// (double-buffered factors, one barrier per batch).
+// point and 128 x 128 tile on the VALU.  VALU instructions can issue while a BF16
+// MFMA runs (not while an FP32 one does, whose 155 TFLOP/s this form beats), so one
+// workgroup of 8 waves per CU, two per SIMD, and in each wave's stream the next
+// batch's generation alternates, slot by slot, with this batch's products
+// (double-buffered factors, one barrier per batch).  By the counters below the two
+// hardly overlap all the same: what the alternation gains is the waits.
 // Fresnel, 100k points at 3840x2160: 94-99 -> 32-34 ms (24.3 without the
 // generation; FP32 MFMA 60, 4 waves without the alternation 40); RS, 20k points
 // (rank 2): 30-31 -> 13.7-14.2 ms (7.7 without it; FP32 MFMA 27.5); 22k points at

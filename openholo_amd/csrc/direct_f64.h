@@ -9,8 +9,10 @@
 // Fresnel, 20k points at 3840x2160: 48.6 -> 23.5 ms (19.4 of them products); RS,
 // 10k points at 1920x1080: 19.1 -> 11.2 ms.  The scalar form read one row factor
 // from LDS per 4 FMAs and wave (Fresnel) and spent 23 FP64 instructions per pair
-// (RS).  128 x 64 pixels is the largest tile whose sums fit 256 registers with two
-// workgroups per CU.
+// (RS).  Two workgroups of 4 waves on 128 x 64 pixels per CU, 128 registers of sums a
+// lane: while one generates, the other multiplies.  (One of 8 waves on 128 x 128
+// would hold the same sums and generate a third less, without a second workgroup to
+// fill its barriers; not measured.)
 #pragma once
 
 namespace dgemm {

@@ -60,8 +60,8 @@ __device__ inline float sin_rev(float x) { return __builtin_amdgcn_sinf(x); }
 __device__ inline float cos_rev(float x) { return __builtin_amdgcn_cosf(x); }
 
 // Points per FP32 partial sum of the FP32 direct kernels, which are folded into
-// FP64 at these boundaries: a point slice that is a whole number of them sums
-// exactly as the one-shot launch does.
+// FP64 at these boundaries, counted from point 0: a point slice that is a whole
+// number of them sums exactly as the one-shot launch does.
 constexpr int DIRECT_CHUNK = 240, DIRECT_CELL = 30;   // see direct_chunk
 
 // Per-point constants produced by the prep kernel (structure of arrays).
@@ -166,8 +166,8 @@ __device__ inline bool rs_mask_bit(const unsigned* __restrict__ row, int t)
 // RS in FP32, whole cloud: the per-pixel kernel alone.  Its 64 x 32 tiles start
 // and end sooner than the matrix kernel's, and points near enough for rank 4 take
 // the same time per pair in either (300 points at 640 x 360: 78 us against 92;
-// at rank 2 77 against 74); with fewer tiles than half the CUs (500 points at 320 x 180:
-// 114 us against 79) or more pairs the matrix kernel is faster.
+// at rank 2 77 against 74); with fewer than 96 tiles (500 points at 320 x 180, 30
+// tiles: 114 us against 79) or more pairs the matrix kernel is faster.
 inline bool direct_per_pixel(const Geometry& g, int64_t n)
 {
     const int64_t tiles = (int64_t)((g.pn_x + 63) / 64) * ((g.pn_y + 31) / 32);

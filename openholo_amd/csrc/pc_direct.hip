@@ -21,8 +21,9 @@
 //  * k_pc_lines adds the one-pixel edge lines of the RS boxes, where the range
 //    test is open.
 //  * k_pc_rest evaluates the RS pairs that the products do not take (points near
-//    the hologram), pixel by pixel on 64 x 32 tiles, one lane per column and 8 rows
-//    per lane: FP64 mode every term; FP32 mode (rest_tile) by point class --
+//    the hologram), pixel by pixel on 64 x 32 tiles (FP64, few of them: 64 x 8, the
+//    points shared by 16 waves), one lane per column and 8 rows per lane: FP64 mode
+//    every term; FP32 mode (rest_tile) by point class --
 //    FAST (whole tile inside the mask, with margin), MASKED (per-pixel mask) or
 //    EXACT (FP32 series not accurate enough: FP64 terms) -- with FP32 constants
 //    recentred on the tile centre, so that no phase exceeds ~65 cycles:
@@ -1196,8 +1197,8 @@ int launch_direct_with(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, dou
     }
     SplitArgs sa{(int)tiles, soa.n, nullptr, chunk};
     if (splits > 1) {
-        // split boundaries on chunk boundaries: a split sums exactly as the
-        // serving engine's point slices do
+        // split boundaries on chunk boundaries: an FP32 split sums exactly as the
+        // serving engine's point slices do (FP64 ones to rounding)
         const int64_t per = (soa.n + splits - 1) / splits;
         sa.split_pts = (per + chunk - 1) / chunk * chunk;
         splits = (int)((soa.n + sa.split_pts - 1) / sa.split_pts);
