@@ -235,7 +235,11 @@ int direct_chunk(const Geometry& g, int64_t n);
 int wrp_generate(ohx_ctx* ctx, const void* d_vertices, int64_t n, const ohx_wrp_params* p, double* d_field,
                  double* d_wrp);
 void wrp_release(ohx_ctx* ctx);
-int launch_direct_jobs(hipStream_t stream, DirectJob* d_jobs, const int* d_njobs);
+// kinds: the kernels that the table's jobs need: jobs_gemm() of those the matrix
+// kernels have tiles of, JOBS_REST if any is RS
+enum : unsigned { JOBS_REST = 16, JOBS_ALL = 31 };
+constexpr unsigned jobs_gemm(int diff, int fp64) { return 1u << (2 * diff + fp64); }
+int launch_direct_jobs(hipStream_t stream, DirectJob* d_jobs, const int* d_njobs, unsigned kinds);
 int launch_fresnel_gemm_range(hipStream_t stream, void* scratch, size_t scratch_bytes, const Geometry& g,
                               const PointSoA& soa, int64_t p0, int64_t p1, double* d_field, uint32_t mode);
 size_t fresnel_gemm_scratch_bytes(const Geometry& g, int64_t npoints);

@@ -1229,18 +1229,22 @@ int direct_tiles(const Geometry& g, bool fp64, int* tiles_x)
     return *tiles_x * ((g.pn_y + gh - 1) / gh);
 }
 
-int launch_direct_jobs(hipStream_t stream, DirectJob* d_jobs, const int* d_njobs)
+int launch_direct_jobs(hipStream_t stream, DirectJob* d_jobs, const int* d_njobs, unsigned kinds)
 {
-    // one workgroup (FP32) or two (FP64) per CU; each returns where the table
-    // holds no job of its kind
+    // one workgroup (FP32) or two (FP64) per CU; a kernel without work returns, but
+    // costs its 4 us in the stream
     constexpr int T32 = dgemm::Kind<float>::NTH, T64 = dgemm::Kind<double>::NTH;
-    hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_RS, float>), dim3(256), dim3(T32), 0, stream, d_jobs, d_njobs);
-    hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_FRESNEL, float>), dim3(256), dim3(T32), 0, stream, d_jobs, d_njobs);
-    hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_RS, double>), dim3(512), dim3(T64), 0, stream, d_jobs, d_njobs);
-    hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_FRESNEL, double>), dim3(512), dim3(T64), 0, stream, d_jobs,
-                       d_njobs);
-    hipLaunchKernelGGL(k_pc_lines_jobs, dim3(1024), dim3(NT), 0, stream, d_jobs, d_njobs);
-    hipLaunchKernelGGL(k_pc_rest_jobs, dim3(512), dim3(NT), 0, stream, d_jobs, d_njobs);
+    constexpr unsigned rs = jobs_gemm(OHX_DIFF_RS, 0) | jobs_gemm(OHX_DIFF_RS, 1);
+    if (kinds & jobs_gemm(OHX_DIFF_RS, 0))
+        hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_RS, float>), dim3(256), dim3(T32), 0, stream, d_jobs, d_njobs);
+    if (kinds & jobs_gemm(OHX_DIFF_FRESNEL, 0))
+        hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_FRESNEL, float>), dim3(256), dim3(T32), 0, stream, d_jobs, d_njobs);
+    if (kinds & jobs_gemm(OHX_DIFF_RS, 1))
+        hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_RS, double>), dim3(512), dim3(T64), 0, stream, d_jobs, d_njobs);
+    if (kinds & jobs_gemm(OHX_DIFF_FRESNEL, 1))
+        hipLaunchKernelGGL((k_pc_gemm_jobs<OHX_DIFF_FRESNEL, double>), dim3(512), dim3(T64), 0, stream, d_jobs, d_njobs);
+    if (kinds & rs) hipLaunchKernelGGL(k_pc_lines_jobs, dim3(1024), dim3(NT), 0, stream, d_jobs, d_njobs);
+    if (kinds & JOBS_REST) hipLaunchKernelGGL(k_pc_rest_jobs, dim3(512), dim3(NT), 0, stream, d_jobs, d_njobs);
     return hipGetLastError() == hipSuccess ? OHX_OK : OHX_ERR_DEVICE;
 }
 

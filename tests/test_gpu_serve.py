@@ -187,3 +187,32 @@ def test_rs_matrix_core_job_without_matrix_core_points():
         st, _, f_direct, _ = srv.wait(srv.submit(v, p, 0, FP32, want_field=True), 120)
         assert st == capi.OK
     assert rel_l2(f_mfma, f_direct) < 1e-12
+
+
+@pytest.mark.parametrize("use_graph", [True, False])
+def test_direct_jobs_of_every_kind(use_graph):
+    """Tables of one formula and precision, RS in FP32 for the per-pixel kernel
+    alone (640x360, 100 points) and points left to it, each alone and all in one
+    burst: as the one-shot launch, to its bar, and alike in the mix."""
+    fp64, fp32 = capi.MODE_GPU, capi.MODE_GPU | capi.MODE_FLOAT
+    kinds = [((640, 360), 100, (0.3, 0.4), 0, fp32), ((300, 200), 400, (0.1, 0.2), 0, fp32),
+             ((300, 200), 400, (0.01, 0.03), 0, fp32), ((300, 200), 400, (0.1, 0.2), 0, fp64),
+             ((300, 200), 400, (0.01, 0.03), 0, fp64), ((300, 200), 400, (0.1, 0.2), 1, fp32),
+             ((300, 200), 400, (0.1, 0.2), 1, fp64)]
+    pp, lam = (8e-6, 8e-6), 532e-9
+    jobs = [(synth.random_cloud(900 + i, n, 1e-3, z), capi.params(pn, pp, lam), diff, mode)
+            for i, (pn, n, z, diff, mode) in enumerate(kinds)]
+    with capi.Server(0, use_graph=use_graph) as srv:
+        alone = []
+        for v, p, diff, mode in jobs:
+            st, _, f, _ = srv.wait(srv.submit(v, p, diff, mode))
+            assert st == capi.OK
+            alone.append(f)
+        ids = [srv.submit(*j) for j in jobs for _ in range(2)]
+        for k, i in enumerate(ids):
+            st, _, f, _ = srv.wait(i)
+            assert st == capi.OK and np.array_equal(f, alone[k // 2]), kinds[k // 2]
+    with capi.Context(0) as ctx:
+        for (pn, n, z, diff, mode), (v, _, _, _), f in zip(kinds, jobs, alone):
+            want = capi.generate(ctx, v, pn, pp, [lam], diff, mode)[0].ravel()
+            assert np.linalg.norm(f - want) <= (1e-11 if mode == fp64 else 1e-6) * np.linalg.norm(want), (z, diff, mode)
