@@ -6,8 +6,8 @@
 // comes on top: FP64 MFMA and any VALU instruction do not issue side by side
 // (measured: a wave of MFMAs and one of FMAs on a SIMD take the sum of their
 // times).
-// Fresnel, 20k points at 3840x2160: 48.6 -> 23.5 ms (19.4 of them products); RS,
-// 10k points at 1920x1080: 19.1 -> 11.2 ms.  The scalar form read one row factor
+// Fresnel, 20k points at 3840x2160: 48.6 -> 23.3 ms (19.4 of them products); RS,
+// 10k points at 1920x1080: 19.1 -> 11.1 ms.  The scalar form read one row factor
 // from LDS per 4 FMAs and wave (Fresnel) and spent 23 FP64 instructions per pair
 // (RS).  Two workgroups of 4 waves on 128 x 64 pixels per CU, 128 registers of sums a
 // lane: while one generates, the other multiplies.  (One of 8 waves on 128 x 128
@@ -28,15 +28,36 @@ constexpr int NLIST = 256;              // listed points of a chunk, each rank's
 struct Smem64 {
     double v[64][ROWD], u[GW][ROWD];    // slot s, point i of it: re at s * 4 + i, im at s * 4 + 2 + i
     double2 tab[NTAB];                  // (cos, sin)(2 pi i / NTAB)
+    double off[2][GW];                  // RS: each column's, row's distance from the tile's centre
     double c[6][NLIST];
     unsigned box[NLIST];                // rows [b0, b1), columns [b2, b3) of the tile, byte k = bk
     int cnt[2][NT / 64][Kind<double>::RMAX + 1];   // [chunk parity][wave][rank]
     int left[2];                        // pairs, box edge lines of pairs left to the per-pixel kernel
 };
 
+// (cos, sin)(2 pi (a b + c) / NTAB), the product unrounded, c in [0, NTAB] (none: 0).
+// The nearest whole number of steps is what the sum with 1.5 2^52 keeps, in its low
+// word the table's index (reduced by a floor first, with the index converted: Fresnel
+// 23.5 ms at 20k points, 3840x2160, now 23.3).
+template <bool C>
+__device__ inline void cis(double a, double b, double c, const double2* tab, double& cs, double& sn)
+{
+    constexpr double whole = 6755399441055744.0;
+    const double s = fma(a, b, whole);
+    int i = __double2loint(s);
+    double r = fma(a, b, whole - s);
+    if (C) {
+        r += c;
+        const double s1 = r + whole;
+        i += __double2loint(s1);
+        r -= s1 - whole;
+    }
+    sincos_step(i, r * (TWO_PI / NTAB), tab, sn, cs);
+}
+
 // Fresnel factors of one batch (listed points j0 .. j0 + n - 1): thread = one
 // point and every 16th column and row, each factor from its own phase.  (Factors
-// advanced by rotations, 20k points at 3840x2160, 22.9 ms against 23.7: but their
+// advanced by rotations, 20k points at 3840x2160, 22.9 ms against 23.3: but their
 // angles are rounded at the size of a step's phase, tens of cycles for a point
 // near the hologram, which left the field off by 1.5e-13 to 3.5e-13 at all
 // depths from 1 mm; by 6e-16 (1 mm) to 1.6e-13 (0.3 m) with phases of their own.)
@@ -47,21 +68,20 @@ __device__ inline void gen_fresnel(Smem64& sm, const Geometry& g, int j0, int n,
     if (p >= n) return;
     const int j = j0 + p, at = (p >> 1) * 4 + (p & 1);
     const unsigned box = sm.box[j];
-    const double q = sm.c[F_Q][j];
+    const double q = sm.c[F_Q][j] * NTAB;
 #pragma unroll
     for (int side = 0; side < 2; ++side) {
         const bool rows = side == 1;
         const unsigned lo = (rows ? box : box >> 16) & 255u, hi = (rows ? box >> 8 : box >> 24) & 255u;
-        const double at0 = sm.c[rows ? F_PY : F_PX][j], cyc = sm.c[F_CYC][j], amp = rows ? sm.c[F_AMP][j] : 1.0;
+        const double at0 = sm.c[rows ? F_PY : F_PX][j], cyc = sm.c[F_CYC][j] * NTAB, amp = rows ? sm.c[F_AMP][j] : 1.0;
         double* dst = (rows ? sm.v[grp] : sm.u[grp]) + at;
 #pragma unroll
         for (int i = 0; i < (rows ? 64 : GW) / NG; ++i) {
             const unsigned k = grp + NG * i;
             const double d = (rows ? pix_y(g, y0 + k) : pix_x(g, x0 + k)) - at0;
-            // mod 1 of the unrounded last product
-            const double qd = q * d, t = fma(qd, d, -floor(qd * d));
             double c, s;
-            sincos2pi(rows ? t + cyc : t, sm.tab, s, c);
+            if (rows) cis<true>(q * d, d, cyc, sm.tab, c, s);
+            else cis<false>(q * d, d, 0.0, sm.tab, c, s);
             const double a = k >= lo && k < hi ? amp : 0.0;
             dst[NG * i * ROWD] = a * c;
             dst[NG * i * ROWD + 2] = a * s;
@@ -72,7 +92,7 @@ __device__ inline void gen_fresnel(Smem64& sm, const Geometry& g, int j0, int n,
 // RS factors of one batch (listed points j0 .. j0 + m - 1 of rank R, unit u into
 // slots u R .. u R + R - 1): thread = one of n >= m points (n a power of two)
 // and every (NT / n)-th column and row.
-__device__ inline void gen_rs(Smem64& sm, const Geometry& g, int j0, int m, int n, int R, int tid, int x0, int y0)
+__device__ inline void gen_rs(Smem64& sm, int j0, int m, int n, int R, int tid)
 {
     const int p = tid & (n - 1), grp = tid / n, NG = NT / n;
     if (p >= m) return;
@@ -83,21 +103,19 @@ __device__ inline void gen_rs(Smem64& sm, const Geometry& g, int j0, int m, int 
         const bool rows = side == 1;
         const unsigned lo = (rows ? box : box >> 16) & 255u, hi = (rows ? box >> 8 : box >> 24) & 255u;
         const double g2 = sm.c[rows ? R_G2Y : R_G2X][j];
-        const double wc = rows ? pix_y(g, y0 + 32) : pix_x(g, x0 + GW / 2);
-        const double cyc = sm.c[R_CYC][j], amp = rows ? sm.c[R_AMP][j] : 1.0;
-        const double ir = sm.c[R_IR][j], rho = sm.c[R_RHO][j];
+        const double cyc = sm.c[R_CYC][j] * NTAB, amp = rows ? sm.c[R_AMP][j] : 1.0;
+        const double ir = sm.c[R_IR][j], rho = sm.c[R_RHO][j], steps = rho * NTAB;
 #pragma unroll 1
         for (int k0 = grp; k0 < (rows ? 64 : GW); k0 += NG) {
-            const double d = (rows ? pix_y(g, y0 + k0) : pix_x(g, x0 + k0)) - wc;
+            const double d = sm.off[side][k0];
             const double e = d * (g2 + d) * ir;
             // sqrt(1 + e) - 1
             const double t =
                 e * fma(e, fma(e, fma(e, fma(e, fma(e, -21.0 / 1024.0, 7.0 / 256.0), -5.0 / 128.0), 1.0 / 16.0), -0.125),
                         0.5);
-            // mod 1 of the unrounded product
-            const double ph = fma(rho, t, -floor(rho * t));
             double c, s;
-            sincos2pi(rows ? ph + cyc : ph, sm.tab, s, c);
+            if (rows) cis<true>(steps, t, cyc, sm.tab, c, s);
+            else cis<false>(steps, t, 0.0, sm.tab, c, s);
             double a = amp * pure_amp<double>(e);
             a = ((unsigned)k0 >= lo && (unsigned)k0 < hi) ? a : 0.0;
             double* dst = (rows ? sm.v[k0] : sm.u[k0]) + at;
@@ -171,6 +189,10 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
         double sn, cs;
         sincospi(2.0 * i / NTAB, &sn, &cs);
         sm.tab[i] = make_double2(cs, sn);
+    }
+    if (DIFF == OHX_DIFF_RS) {
+        if (tid < GW) sm.off[0][tid] = pix_x(g, x0 + tid) - pix_x(g, x0 + GW / 2);
+        if (tid < GH) sm.off[1][tid] = pix_y(g, y0 + tid) - pix_y(g, y0 + GH / 2);
     }
     if (tid < 2) sm.left[tid] = 0;
     Acc64 acc;
@@ -259,7 +281,7 @@ __device__ __attribute__((always_inline)) inline unsigned tile_sum(Smem64& sm, c
             for (int u0 = 0; u0 < units; u0 += per) {
                 const int nu = min(per, units - u0);
                 if constexpr (DIFF == OHX_DIFF_FRESNEL) gen_fresnel(sm, g, beg + u0 * UN, nu * UN, tid, x0, y0);
-                else gen_rs(sm, g, beg + u0 * UN, nu * UN, per * UN, r, tid, x0, y0);
+                else gen_rs(sm, beg + u0 * UN, nu * UN, per * UN, r, tid);
                 __syncthreads();
                 multiply(sm, acc, nu * r, wave >> 1, wave & 1, lane);
                 __syncthreads();

@@ -202,15 +202,12 @@ __device__ inline void exact_term(double dx, double dy, double z, double cyc0, d
 // FP32 factors and FP32 sums over a chunk, folded into FP64).
 constexpr int NTAB = 256;  // angles of the FP64 sin/cos table
 
-// sin and cos of 2 pi t, t in [0, 2], in FP64: the nearest table angle
-// 2 pi i / NTAB plus Taylor series of the remainder |x| <= pi / NTAB
-// (dropped terms below 2e-20), combined by angle addition; about 17 FP64
-// instructions and one LDS read against ~40 for sincospi.
-__device__ inline void sincos2pi(double t, const double2* __restrict__ tab, double& s, double& c)
+// sin and cos of 2 pi i / NTAB + x, |x| <= pi / NTAB, in FP64: the table's angle
+// plus Taylor series of x (dropped terms below 2e-20), combined by angle addition; 13
+// FP64 instructions and one LDS read against ~40 for sincospi.
+__device__ inline void sincos_step(int i, double x, const double2* __restrict__ tab, double& s, double& c)
 {
-    const double ti = rint(t * NTAB);
-    const double x = fma(ti, -1.0 / NTAB, t) * TWO_PI;
-    const double2 a = tab[(int)ti & (NTAB - 1)];   // (cos, sin)(2 pi i / NTAB)
+    const double2 a = tab[i & (NTAB - 1)];   // (cos, sin)(2 pi i / NTAB)
     const double x2 = x * x;
     const double cb = fma(x2, fma(x2, fma(x2, -1.0 / 720.0, 1.0 / 24.0), -0.5), 1.0);
     const double sb = x * fma(x2, fma(x2, fma(x2, -1.0 / 5040.0, 1.0 / 120.0), -1.0 / 6.0), 1.0);

@@ -120,3 +120,16 @@ def test_rs_fp64_left_points(ctx, pn, n):
 def test_fp64_listed_points(ctx, n, z, diff):
     v = synth.random_cloud(6290 + n, n, 1.5e-3, z, complex_amplitude=True)
     check(ctx, v, (300, 200), (8e-6, 8e-6), diff, FP64, 1e-11, use_phase=True)
+
+
+# Fresnel points so far away that their phases have no digits left: finite, and as
+# in the probe
+@pytest.mark.parametrize("mode", [FP64, FP32])
+@pytest.mark.parametrize("x,z", [(1e3, 1e6), (1e12, 1e18), (1e80, 1e90), (1e150, 1e160)])
+def test_fresnel_far_points(ctx, x, z, mode):
+    v = synth.random_cloud(6295, 3, 1e-3, (0.1, 0.2)).copy()
+    v["pos"][1] = x, -0.5 * x, z
+    pn, pp = (200, 100), (8e-6, 8e-6)
+    got = capi.generate(ctx, v[1:2], pn, pp, [LAM], 1, mode)[0].ravel()
+    assert np.isfinite(got).all() and (got != 0).any()
+    check(ctx, v, pn, pp, 1, mode, 1e-11 if mode == FP64 else 1e-5)
