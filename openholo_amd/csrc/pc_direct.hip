@@ -1084,7 +1084,10 @@ static double makespan(double first, double c, double tiles, double cl, double s
     return full * c + t;
 }
 
-static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, int chunk, GemmCost k, double* time)
+// masked: the launch skips most pairs (rs_skip_mask) and some tiles hold all of the
+// rest, so its time is that of the longest workgroup after a quarter of the whole work.
+static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, int chunk, GemmCost k, bool masked,
+                             double* time)
 {
     int best = 1;
     for (int S = 1; S <= MAX_SPLITS; ++S) {
@@ -1092,9 +1095,10 @@ static int gemm_point_splits(int64_t tiles, int64_t n, int slots, int64_t npx, i
                       tiles * (S - 1) > 8 * (int64_t)slots))
             break;
         const int64_t per = S == 1 ? n : ((n + S - 1) / S + chunk - 1) / chunk * chunk, parts = (n + per - 1) / per;
-        const double t = makespan((double)(tiles * (parts - 1)), per * k.point + k.tile, (double)tiles,
-                                  (n - (parts - 1) * per) * k.point + k.tile, slots) +
-                         (parts > 1 ? 40.0 + (parts - 1) * (npx * 8e-5) : 0.0);
+        const double c = per * k.point + k.tile, cl = (n - (parts - 1) * per) * k.point + k.tile;
+        const double run = masked ? c + (double)tiles * (n * k.point * 0.25 + parts * k.tile) / slots
+                                  : makespan((double)(tiles * (parts - 1)), c, (double)tiles, cl, slots);
+        const double t = run + (parts > 1 ? 40.0 + (parts - 1) * (npx * 8e-5) : 0.0);
         // the first further plane by a tenth, for the model takes every box as whole
         if (S == 1 || t < *time * (best == 1 ? 0.9 : 0.97)) {
             best = S;
@@ -1121,7 +1125,7 @@ int direct_chunk(const Geometry& g, int64_t n)
     double best_t = 0.0;
     for (int first = best, chunk = first; chunk >= least; chunk /= 2) {
         double t;
-        gemm_point_splits(tiles, n, 256, npx, chunk, gemm_cost(rs, false, chunk), &t);
+        gemm_point_splits(tiles, n, 256, npx, chunk, gemm_cost(rs, false, chunk), false, &t);
         if (chunk == first || t < best_t * 0.9) {
             best = chunk;
             best_t = t;
@@ -1190,7 +1194,7 @@ int launch_direct_with(ohx_ctx* ctx, const Geometry& g, const PointSoA& soa, dou
         double t;
         splits = gemm_point_splits(tiles, soa.n,
                                    resident_slots(ctx, kern, fp64 ? dgemm::Kind<double>::NTH : dgemm::Kind<float>::NTH),
-                                   npx, chunk, gemm_cost(rs, fp64, chunk), &t);
+                                   npx, chunk, gemm_cost(rs, fp64, chunk), g.rs_skip_mask != nullptr, &t);
     }
     SplitArgs sa{(int)tiles, soa.n, nullptr, chunk};
     if (splits > 1) {
